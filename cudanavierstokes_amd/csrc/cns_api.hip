@@ -384,12 +384,6 @@ static void build_grid(cns_solver *s) {
                                    s->cVF[2 * SV - it] * xpp[i] * (xp[i] * xp[i] * xp[i]) * s->d_dx);
 }
 
-// Workgroup grid of the stage kernels: x-y tiles (tile_x() x 16 columns)
-// times z chunks of zc planes.  Default chunk length (measured on 256^3 and
-// 128^3 Taylor-Green cases): the FP64 kernel (one workgroup per CU) prefers
-// long marches, about one workgroup per CU, chunks of 8..256 planes, and so
-// does the FP32 kernel with mu = T/Re (one 512-lane workgroup per CU); small
-// grids want chunks of 8.  cns_tune measures instead.
 static void set_pencil(cns_solver *s, int zc) {
     const cns_config &c = s->cfg;
     zc = std::max(1, std::min(zc, c.nz));
@@ -407,26 +401,49 @@ static void set_pencil(cns_solver *s, int zc) {
     s->base.nzc = s->nzc;
 }
 
+// Workgroup grid of the stage kernels: x-y tiles (tile_x() x 16 columns)
+// times z chunks of zc planes.  One RHS workgroup runs on a CU at a time
+// (512 lanes at two waves per SIMD), and each of the 8 XCDs works through a
+// contiguous eighth of the grid on its 32 CUs (remap_block), so a launch
+// takes rounds x (zc + fill) plane times, rounds = ceil(workgroups / 8 / 32)
+// and fill about two planes for the window's first loads (fitted on
+// 24^3..256^3 boxes and channels, orders 4-8, both precisions, pencils
+// 1..256: 1.4-3 us a plane, fill 1-2.3 planes).  The default chunk count is
+// the one with the fewest plane times, the smaller count of equals.  Against
+// one workgroup per CU whatever the XCDs' shares (chunks of 8..256 planes):
+// the 160x128x192 order-6 channel, 4 chunks -> 3, 346 -> 202 us per launch;
+// 64^3 order 4, 8 -> 16 chunks, 22.5 -> 17.0 us; 24^3 order 6, 3 -> 24
+// chunks, 23.9 -> 12.1 us; FP32 channel, 13 -> 6 chunks, 229 -> 165 us;
+// 272x240x256, 2 -> 1 chunks, 1297 -> about 770 us.  cns_tune measures.
+static int default_pencil(long cols, int nz) {
+    const long xcds = 8, cus = 32, fill = 2;
+    int best = nz;
+    long cost = 0;
+    for (int nzc = 1; nzc <= nz; nzc++) {
+        const int zc = (nz + nzc - 1) / nzc;
+        const long share = (cols * ((nz + zc - 1) / zc) + xcds - 1) / xcds;
+        const long c = (share + cus - 1) / cus * (zc + fill);
+        if (nzc == 1 || c < cost) {
+            cost = c;
+            best = zc;
+        }
+    }
+    return best;
+}
+
 static void launch_geometry(cns_solver *s) {
     const cns_config &c = s->cfg;
     const bool fp32 = c.precision == CNS_FP32, unitv = c.visc_exp == 1.0;
     const int tx = tile_x_of(fp32, unitv);
     s->ntx = (c.nx + tx - 1) / tx;
     s->nty = (c.ny + TILE_Y - 1) / TILE_Y;
-    const long cols = (long)s->ntx * s->nty;
-    // workgroups to aim at: one round, i.e. one 512-lane workgroup per CU at
-    // two waves per SIMD, or two rounds of shorter marches for FP32 with a
-    // general viscosity law (measured faster there)
-    const long target = (fp32 && !unitv) ? 512 : 256;
-    long zc = ((long)c.nz * cols + target - 1) / target;
-    zc = std::max<long>(zc, 8);
-    zc = std::min<long>(zc, 256);
+    int zc = default_pencil((long)s->ntx * s->nty, c.nz);
     // CNS_PENCIL=<planes>: z-chunk length override
     if (const char *pz = std::getenv("CNS_PENCIL")) {
         const int v = std::atoi(pz);
         if (v >= 1) zc = v;
     }
-    set_pencil(s, (int)zc);
+    set_pencil(s, zc);
 }
 
 static void fill_params(cns_solver *s) {
