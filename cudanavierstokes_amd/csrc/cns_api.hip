@@ -1714,13 +1714,13 @@ static int xprof_t(cns_solver *s, double *prof) {
     // chunk partials in the first rhs set (free between steps):
     // nch * 5 * mx doubles within its 5 * n * esz bytes
     double *part = static_cast<double *>(s->rbuf[0]);
-    const int nch = (int)std::max(1L, std::min(256L, rows * (long)s->esz / 8));
-    const dim3 grid((mx + 255) / 256, nch), fin((mx + 255) / 256);
+    const int nch = (int)std::max(1L, std::min((long)PROF_CHUNKS, rows * (long)s->esz / 8));
+    const dim3 grid((mx + 255) / 256, nch), fin((mx + 63) / 64);
     for (int pass = 0; pass < 2; pass++) {
         hipLaunchKernelGGL(k_xprof_sums<R>, grid, dim3(256), 0, s->stream, mx, rows, (long)s->n, q, lo, s->rho0, s->E0,
                            pass, (const double *)s->d_prof, part, nch);
         LAUNCHED(s, "k_xprof_sums");
-        hipLaunchKernelGGL(k_xprof_final, fin, dim3(256), 0, s->stream, mx, my, mz, (const double *)part, nch, pass,
+        hipLaunchKernelGGL(k_xprof_final, fin, dim3(64 * PROF_GROUPS), 0, s->stream, mx, my, mz, (const double *)part, nch, pass,
                            s->d_prof);
         LAUNCHED(s, "k_xprof_final");
     }
