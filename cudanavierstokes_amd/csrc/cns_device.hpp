@@ -171,16 +171,92 @@ __device__ __forceinline__ int remap_block(int b, int nb, int on) {
     return start + slot;
 }
 
-// T^n of the FP64 viscosity law mu = T^n / Re (T > 0): T sqrt(T) for the
-// boundary layer's n = 3/2, else exp2(n log2 T); both within a few ulp of
-// pow(T, n) at 7% and 60% of its instructions (pow handles every sign and
-// special case of its arguments, which a temperature never needs).
-__device__ __forceinline__ double visc_pow(double t, double n) { return n == 1.5 ? t * sqrt(t) : exp2(n * log2(t)); }
+// T^n of the FP64 viscosity law mu = T^n / Re: T sqrt(T) for the boundary
+// layer's n = 3/2, else 2^(n log2 T) from two series evaluated here, the
+// column role's longest piece of arithmetic on a general-viscosity flow (two
+// a point; the plane role waited 26% of its time for the column role):
+//   T = m 2^e, m in [sqrt(1/2), sqrt(2)),  f = (m - 1)/(m + 1),
+//   log2 m = (2/ln 2) (f + f^3/3 + ... + f^21/21)       (|f| <= 0.172)
+//   2^r = sum_{k <= 13} (r ln 2)^k / k!                  (|r| <= 1/2)
+// whose remainders are below 3e-17 relative.  The powers are formed first and
+// the series summed as two chains: a coefficient is then a multiplier, which
+// an instruction takes from scalar registers, and not an addend to move into
+// vector registers (two moves each).  The leading terms of the logarithm are
+// carried in two doubles, so the result is within 1.2 ulp of T^n whatever n log2 T
+// (exp2(n log2 T): 1 ulp and the exponent's rounding, 6 ulp at T^2 = 0.004;
+// tests/test_visc_pow.py), at about 95 vector instructions instead of 158.  A T
+// that is no positive finite number goes through exp2 and log2 themselves.
+__device__ __forceinline__ double pow_series(double t, double n) {
+#ifdef __clang__
+#pragma clang fp contract(off)  // the low parts below need their products rounded
+#endif
+    int e;
+    double m = frexp(t, &e);
+    const bool low = m < 0.70710678118654752440;
+    m = low ? 2.0 * m : m;
+    e = low ? e - 1 : e;
+    // 2/ln 2 = C + CL; f + fl = (m - 1)/(m + 1) beyond double precision
+    constexpr double L = 0.69314718055994530942, C = 2.8853900817779268, CL = 4.0710547481862064e-17;
+    const double d = m + 1.0, g = m - 1.0, i = 1.0 / d, f = g * i;
+    const double fl = fma(-f, m - (d - 1.0), fma(-f, d, g)) * i;
+    const double s = f * f, s2 = s * s, s3 = s2 * s, s4 = s2 * s2, s5 = s3 * s2, s6 = s3 * s3, s7 = s4 * s3,
+                 s8 = s4 * s4, s9 = s5 * s4, s10 = s5 * s5;
+    double a = (C / 21.0) * s10, b = (C / 19.0) * s9;
+    a = fma((C / 17.0), s8, a);
+    b = fma((C / 15.0), s7, b);
+    a = fma((C / 13.0), s6, a);
+    b = fma((C / 11.0), s5, b);
+    a = fma((C / 9.0), s4, a);
+    b = fma((C / 7.0), s3, b);
+    a = fma((C / 5.0), s2, a);
+    b = fma((C / 3.0), s, b);
+    // log2 T = lh + ll and n log2 T = yh + yl, each low part what the rounding
+    // of its high part left (|C f| <= 1/2, so e leads the sum unless it is 0)
+    const double hi = C * f, ed = (double)e, lh = ed + hi;
+    const double ll = (hi - (lh - ed)) + fma(f, a + b, fma(C, f, -hi) + fma(C, fl, CL * f));
+    const double yh = n * lh, yl = fma(n, ll, fma(n, lh, -yh));
+    const double k = rint(yh), r = (yh - k) + yl;
+    constexpr double L2 = L * L, L3 = L2 * L, L4 = L2 * L2, L5 = L3 * L2, L6 = L3 * L3, L7 = L4 * L3;
+    const double r2 = r * r, r3 = r2 * r, r4 = r2 * r2, r5 = r3 * r2, r6 = r3 * r3, r7 = r4 * r3, r8 = r4 * r4,
+                 r9 = r5 * r4, r10 = r5 * r5, r11 = r6 * r5, r12 = r6 * r6, r13 = r7 * r6;
+    double u = (L6 * L6 / 479001600.0) * r12, v = (L7 * L6 / 6227020800.0) * r13;
+    u = fma((L5 * L5 / 3628800.0), r10, u);
+    v = fma((L6 * L5 / 39916800.0), r11, v);
+    u = fma((L4 * L4 / 40320.0), r8, u);
+    v = fma((L5 * L4 / 362880.0), r9, v);
+    u = fma((L6 / 720.0), r6, u);
+    v = fma((L7 / 5040.0), r7, v);
+    u = fma((L4 / 24.0), r4, u);
+    v = fma((L5 / 120.0), r5, v);
+    u = fma((L2 / 2.0), r2, u);
+    v = fma((L3 / 6.0), r3, v);
+    return ldexp(1.0 + (u + fma(L, r, v)), (int)k);
+}
 
-// Equation of state and viscosity law (src/cuda_main.cu:228-239).
-template <typename R, bool UNITV>
-__device__ __forceinline__ void eos(const Params &P, R r, R ru, R rv, R rw, R re, R &u, R &v, R &w, R &t,
-                                    R &h, R &mu) {
+__device__ __forceinline__ bool pow_regular(double t) { return t > 0.0 && t < HUGE_VAL; }
+__device__ __forceinline__ double visc_pow(double t, double n) {
+    if (n == 1.5) return t * sqrt(t);
+    return pow_regular(t) ? pow_series(t, n) : exp2(n * log2(t));
+}
+// two at once: one block of instructions in which the chains of the two
+// series hide each other's latency
+__device__ __forceinline__ void visc_pow2(double t0, double t1, double n, double &p0, double &p1) {
+    if (n == 1.5) {
+        p0 = t0 * sqrt(t0);
+        p1 = t1 * sqrt(t1);
+    } else if (pow_regular(t0) && pow_regular(t1)) {
+        p0 = pow_series(t0, n);
+        p1 = pow_series(t1, n);
+    } else {
+        p0 = exp2(n * log2(t0));
+        p1 = exp2(n * log2(t1));
+    }
+}
+
+// Equation of state (src/cuda_main.cu:228-237); mu = T^viscexp / Re follows
+// from the final T (to_prim), for viscexp = 1 the kernels rebuild it as T/Re.
+template <typename R>
+__device__ __forceinline__ void eos(const Params &P, R r, R ru, R rv, R rw, R re, R &u, R &v, R &w, R &t, R &h) {
     R inv = R(1) / r;
     u = ru * inv;
     v = rv * inv;
@@ -190,21 +266,18 @@ __device__ __forceinline__ void eos(const Params &P, R r, R ru, R rv, R rw, R re
     t = R(P.cvInv) * en;
     // total enthalpy (rhoE + p)/rho = cp T + |u|^2/2 with cp = gam R/(gam-1)
     h = t * R(P.cpR) + k2;
-    // mu = T^viscexp / Re; for viscexp = 1 the kernels rebuild it as T/Re
-    mu = UNITV ? R(0) : R(visc_pow((double)t, P.viscexp)) * R(P.invRe);
 }
 
 // Isothermal no-slip wall ghost from its mirror point (src/boundary.h:79-148):
 // velocity antisymmetric, pressure and dilatation symmetric, T = 2Tw - T,
-// mu and lambda from the ghost T, rho = p/(R T), h = cp T + |u|^2/2.
-template <typename R, bool UNITV>
-__device__ __forceinline__ void wall_ghost(const Params &P, R tw, R &r, R &u, R &v, R &w, R &t, R &h, R &mu) {
+// rho = p/(R T), h = cp T + |u|^2/2 (mu and lambda from the ghost T: to_prim).
+template <typename R>
+__device__ __forceinline__ void wall_ghost(const Params &P, R tw, R &r, R &u, R &v, R &w, R &t, R &h) {
     R p = r * R(P.Rgas) * t;
     u = -u;
     v = -v;
     w = -w;
     t = R(2.0) * tw - t;
-    mu = UNITV ? R(0) : R(visc_pow((double)t, P.viscexp)) * R(P.invRe);
     h = t * R(P.cpR) + R(0.5) * (u * u + v * v + w * w);
     r = p / (R(P.Rgas) * t);
 }
@@ -263,9 +336,9 @@ __device__ __forceinline__ float visc_law(float t, float n, float inv_re) {
 //   h' = (E' + p' - rho' h0)/rho,
 // so that T = T0 + T' and h = h0 + h' carry the fluctuation at full relative
 // precision (p0, T0, h0 cancel exactly in the algebra).
-template <typename R, bool UNITV>
+template <typename R>
 __device__ __forceinline__ void eos_off(const Params &P, R rp, R ru, R rv, R rw, R ep, R &u, R &v, R &w, R &tp,
-                                        R &hp, R &mu) {
+                                        R &hp) {
     const R r = R(P.rho0) + rp;
     const R inv = recip(r);
     u = ru * inv;
@@ -275,7 +348,6 @@ __device__ __forceinline__ void eos_off(const Params &P, R rp, R ru, R rv, R rw,
     const R pp = R(P.gam - 1.0) * (ep - r * k2);
     tp = (pp - rp * R(P.Rgas * P.T0)) * inv * R(1.0 / P.Rgas);
     hp = (ep + pp - rp * R(P.h0)) * inv;
-    mu = UNITV ? R(0) : visc_law(R(P.T0) + tp, R(P.viscexp), R(P.invRe));
 }
 
 // Wall ghost on offset storage (FP32), from the mirror point's offsets:
@@ -285,9 +357,8 @@ __device__ __forceinline__ void eos_off(const Params &P, R rp, R ru, R rv, R rw,
 //   h'_g   = cp T'_g + |u|^2/2 + (cp T0 - h0),
 // every term of the size of the fluctuation, so FP32 keeps its relative
 // precision (dtw = Tw - T0 in FP64 on the host).
-template <typename R, bool UNITV>
-__device__ __forceinline__ void wall_ghost_off(const Params &P, R dtw, R &rp, R &u, R &v, R &w, R &tp, R &hp,
-                                               R &mu) {
+template <typename R>
+__device__ __forceinline__ void wall_ghost_off(const Params &P, R dtw, R &rp, R &u, R &v, R &w, R &tp, R &hp) {
     const R T0 = R(P.T0), r0 = R(P.rho0);
     const R t = T0 + tp;
     const R tpg = R(2) * dtw - tp;
@@ -298,7 +369,6 @@ __device__ __forceinline__ void wall_ghost_off(const Params &P, R dtw, R &rp, R 
     w = -w;
     tp = tpg;
     hp = R(P.cpR) * tpg + R(0.5) * (u * u + v * v + w * w) + R(P.ch0);
-    mu = UNITV ? R(0) : visc_law(tg, R(P.viscexp), R(P.invRe));
 }
 
 // Quantity indices of the staged primitives (LDS plane and z register

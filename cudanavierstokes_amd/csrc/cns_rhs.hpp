@@ -85,16 +85,16 @@ __device__ __forceinline__ void load_raw(const StagePtrs<R> &A, long poff, unsig
 
 // Primitives of one loaded point with the x ghost rule of its side applied.
 // On offset storage (FP32) rho, T and h are staged as rho', T', h'.
-template <typename R, bool WALLX, bool UNITV>
-__device__ __forceinline__ void to_prim(const Params &P, const Raw<R> &x, int side, R *q) {
-    R r = x.c[0], u, v, w, t, h, mu;
+// prim_of leaves the viscosity out; to_prim adds it from the final T.
+template <typename R, bool WALLX>
+__device__ __forceinline__ void prim_of(const Params &P, const Raw<R> &x, int side, R *q) {
+    R r = x.c[0], u, v, w, t, h;
     if constexpr (Off<R>::on) {
-        eos_off<R, UNITV>(P, r, x.c[1], x.c[2], x.c[3], x.c[4], u, v, w, t, h, mu);
-        if (WALLX && side != 0) wall_ghost_off<R, UNITV>(P, R(side < 0 ? P.dtw_bot : P.dtw_top), r, u, v, w, t, h, mu);
+        eos_off<R>(P, r, x.c[1], x.c[2], x.c[3], x.c[4], u, v, w, t, h);
+        if (WALLX && side != 0) wall_ghost_off<R>(P, R(side < 0 ? P.dtw_bot : P.dtw_top), r, u, v, w, t, h);
     } else {
-        eos<R, UNITV>(P, r, x.c[1], x.c[2], x.c[3], x.c[4], u, v, w, t, h, mu);
-        if (WALLX && side != 0)
-            wall_ghost<R, UNITV>(P, side < 0 ? R(P.twall_bot) : R(P.twall_top), r, u, v, w, t, h, mu);
+        eos<R>(P, r, x.c[1], x.c[2], x.c[3], x.c[4], u, v, w, t, h);
+        if (WALLX && side != 0) wall_ghost<R>(P, side < 0 ? R(P.twall_bot) : R(P.twall_top), r, u, v, w, t, h);
     }
     q[QR] = r;
     q[QU] = u;
@@ -103,7 +103,25 @@ __device__ __forceinline__ void to_prim(const Params &P, const Raw<R> &x, int si
     q[QH] = h;
     q[QT] = t;
     q[QD] = x.d;
-    q[QM] = mu;
+    q[QM] = R(0);
+}
+template <typename R, bool WALLX, bool UNITV>
+__device__ __forceinline__ void to_prim(const Params &P, const Raw<R> &x, int side, R *q) {
+    prim_of<R, WALLX>(P, x, side, q);
+    if constexpr (!UNITV) {
+        if constexpr (Off<R>::on)
+            q[QM] = visc_law(R(P.T0) + q[QT], R(P.viscexp), R(P.invRe));
+        else
+            q[QM] = R(visc_pow((double)q[QT], P.viscexp)) * R(P.invRe);
+    }
+}
+// The viscosities of two points from their T (FP64), as visc_pow2 does.
+template <typename R>
+__device__ __forceinline__ void add_visc2(const Params &P, R *q0, R *q1) {
+    double p0, p1;
+    visc_pow2((double)q0[QT], (double)q1[QT], P.viscexp, p0, p1);
+    q0[QM] = R(p0) * R(P.invRe);
+    q1[QM] = R(p1) * R(P.invRe);
 }
 
 // Viscous-order first and second derivatives of u, v, w along DIR
@@ -922,25 +940,20 @@ __device__ __forceinline__ void rhs_tile_split(const Params &P, const StagePtrs<
             bcos = cos(((double)wrapi(y0 + hly - H, P.my) / P.d_dy) / P.blow_lam);
         }
     }
-    // the halo point of plane k into LDS buffer b, then the prefetch of
-    // plane k+1; BL: the source point's primitives, at the bottom the
-    // adiabatic reflection with the blowing (the top is formed by top_ghost)
-    auto stage_halo = [&](int k, int b) {
-        R t[NQ];
+    // the halo point of plane k (primitives t of its source point) into LDS
+    // buffer b; BL: at the bottom the adiabatic reflection with the blowing (the
+    // top is formed by top_ghost)
+    auto stage_halo = [&](int k, int b, R *t) {
         if constexpr (BL) {
-            to_prim<R, false, UNITV>(P, hr, 0, t);
             if (hside < 0) {
                 double ub = 0.0;
                 const bool blow = P.perturbed && bl_blow(k, bs1, bs2, bcos, ub);
                 bl_bottom_ghost<R>(P, blow, R(ub), t[QR], t[QU], t[QV], t[QW], t[QT], t[QH]);
             }
-        } else {
-            to_prim<R, WALLX, UNITV>(P, hr, hside, t);
         }
         const int ws = hact ? hslot : 0;
 #pragma unroll
         for (int q = 0; q < NL; q++) sq[b][q][ws] = t[q];
-        load_raw(A, (long)wrap1(k + 1, P.mz) * mxy, hoff, hr);
     };
     // BL: the top x ghost of the halo point from the staged plane (topBCxExt
     // on u, v, w, p, T, dil; rho, h, mu from the ghost p and T:
@@ -978,13 +991,30 @@ __device__ __forceinline__ void rhs_tile_split(const Params &P, const StagePtrs<
             if constexpr (BL) win[NL][a] = t[QR] * R(P.Rgas) * t[QT];
         };
         // unconditional loads (see rhs_tile)
+        if constexpr (UNITV) {
 #pragma unroll
-        for (int a = 0; a < W - 1; a++) {
-            Raw<R> x;
-            load_raw(A, (long)wrap1(z0 - H + a, P.mz) * mxy, coff, x);
-            R t[NQ];
-            to_prim<R, WALLX, UNITV>(P, x, cside, t);
-            push(t, a);
+            for (int a = 0; a < W - 1; a++) {
+                Raw<R> x;
+                load_raw(A, (long)wrap1(z0 - H + a, P.mz) * mxy, coff, x);
+                R t[NQ];
+                to_prim<R, WALLX, UNITV>(P, x, cside, t);
+                push(t, a);
+            }
+        } else {
+            // the viscosity's branches would put each plane's loads behind the
+            // last one's arithmetic: all planes' loads first
+            Raw<R> x[W - 1];
+#pragma unroll
+            for (int a = 0; a < W - 1; a++) load_raw(A, (long)wrap1(z0 - H + a, P.mz) * mxy, coff, x[a]);
+#pragma unroll
+            for (int a = 0; a < W - 1; a += 2) {
+                R t[NQ], t1[NQ];
+                prim_of<R, WALLX>(P, x[a], cside, t);
+                prim_of<R, WALLX>(P, x[a + 1], cside, t1);
+                add_visc2(P, t, t1);
+                push(t, a);
+                push(t1, a + 1);
+            }
         }
         Raw<R> zr;  // prefetched window feed (plane k + H)
         load_raw(A, (long)wrap1(z0 + H, P.mz) * mxy, coff, zr);
@@ -997,6 +1027,28 @@ __device__ __forceinline__ void rhs_tile_split(const Params &P, const StagePtrs<
             const int b = (k - z0) & 1;
             R d1z[3], d2z[3];
             {
+                // The column's point and the halo point together: the chains of
+                // the two equations of state and viscosity series (each with
+                // branches of its own, which the scheduler does not cross)
+                // hide each other's latency, and the next plane's loads are
+                // issued before the series, so that they have the rest of the
+                // plane to arrive.  Per launch against one point after the other
+                // with exp2(n log2 T): order-8 channel 160x128x192 284 -> 223 us,
+                // 101x67x83 order 8/4 56.8 -> 45.3, 90x75x110 order 6/4 53.8 ->
+                // 48.2; order-6 channel and mu = T/Re within 1%.  The boundary
+                // layer (mu = T^1.5/Re has no series) loses 6% by it and takes
+                // one point after the other.
+                R t[NQ], th[NQ];
+                if constexpr (BL) {
+                    to_prim<R, WALLX, UNITV>(P, zr, cside, t);
+                } else {
+                    prim_of<R, WALLX>(P, zr, cside, t);
+                    prim_of<R, WALLX>(P, hr, hside, th);
+                    load_raw(A, (long)wrap1(k + 1 + H, P.mz) * mxy, coff, zr);
+                    load_raw(A, (long)wrap1(k + 1, P.mz) * mxy, hoff, hr);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (!UNITV) add_visc2(P, t, th);
+                }
                 if (BL && k + H >= P.mz) {
                     // top z ghost: f(mz-1+d) = 2 f(mz-1) - f(mz-1-d) (topBCzExt)
                     const int d = k + H - (P.mz - 1);
@@ -1006,8 +1058,6 @@ __device__ __forceinline__ void rhs_tile_split(const Params &P, const StagePtrs<
 #pragma unroll
                             for (int q = 0; q < NW; q++) win[q][W - 1] = R(2) * win[q][W - 1 - dd] - win[q][W - 1 - 2 * dd];
                 } else {
-                    R t[NQ];
-                    to_prim<R, WALLX, UNITV>(P, zr, cside, t);
                     push(t, W - 1);
                 }
                 if (BL && k == 0) {
@@ -1019,8 +1069,12 @@ __device__ __forceinline__ void rhs_tile_split(const Params &P, const StagePtrs<
                 }
 #pragma unroll
                 for (int q = 0; q < NL; q++) sq[b][q][cc] = win[q][H];
-                load_raw(A, (long)wrap1(k + 1 + H, P.mz) * mxy, coff, zr);
-                stage_halo(k, b);
+                if constexpr (BL) {
+                    load_raw(A, (long)wrap1(k + 1 + H, P.mz) * mxy, coff, zr);
+                    to_prim<R, false, UNITV>(P, hr, 0, th);
+                }
+                stage_halo(k, b, th);
+                if constexpr (BL) load_raw(A, (long)wrap1(k + 1, P.mz) * mxy, hoff, hr);
             }
             vel_stencils<R, SV, 2, false>(P, FZ, nullptr, 1.0, d1z, d2z);
             xgz[b][0][tid] = d1z[0];
