@@ -2037,13 +2037,43 @@ static int bfail(cns_batch *b, int code, const std::string &msg) {
     return code;
 }
 
-// z chunks of member m under pencil length L (at least the window depth)
+// z chunks of member m under pencil length L (at least the window depth), of
+// even lengths
 static void member_geometry(const cns_solver *m, int L, int &zc, int &nzc, int &nwork) {
     const int mz = m->cfg.nz;
     const int lo = std::min(2 * m->S, mz);
-    zc = std::max(std::min(L, mz), lo);
+    nzc = (mz + std::max(std::min(L, mz), lo) - 1) / std::max(std::min(L, mz), lo);
+    zc = std::max((mz + nzc - 1) / nzc, lo);
     nzc = (mz + zc - 1) / zc;
     nwork = m->ntx * m->nty * nzc;
+}
+
+// Pencil length of a group whose shape nobody has set: the launch's plane
+// times, rounds x (longest chunk + fill) as in default_pencil, over lengths
+// 4..64 (one workgroup per item on the same CUs, so the same rounds).  Against
+// 16 planes for FP32 (32 for FP64) whatever the members: 12 order-6 RK4 boxes
+// 128^3..32^3 1840 -> 1719 us a step, ten FP32 boxes and channels up to 160^3
+// (16 planes are 33 rounds' worth of the channels' items on 32 CUs) 2058 -> 1930.
+static int default_batch_pencil(const BatchGroup &g) {
+    const long xcds = 8, cus = 32, fill = 2;
+    int best = 16;
+    long cost = 0;
+    for (int L = 4; L <= 64; L++) {
+        long items = 0;
+        int longest = 0;
+        for (const cns_solver *m : g.m) {
+            int zc, nzc, nw;
+            member_geometry(m, L, zc, nzc, nw);
+            items += nw;
+            longest = std::max(longest, zc);
+        }
+        const long c = ((items + xcds - 1) / xcds + cus - 1) / cus * (longest + fill);
+        if (L == 4 || c < cost) {
+            cost = c;
+            best = L;
+        }
+    }
+    return best;
 }
 
 // Jobs of every stage of group g under pencil L.  scratch: the tuning form,
@@ -2257,10 +2287,8 @@ extern "C" int cns_batch_create(cns_solver *const *members, int n, cns_batch **o
             g->scheme = m->cfg.scheme;
             g->nst = n_stages(m);
             // untuned shape: one workgroup per item (the dispatcher balances
-            // members of different sizes); short pencils for FP32 storage,
-            // whose kernels run two workgroups per CU
+            // members of different sizes)
             g->grid = 0;
-            g->pencil = fp32 ? 16 : 32;
         }
         g->m.push_back(m);
         g->forcing = g->forcing || m->cfg.forcing_z;
@@ -2278,6 +2306,7 @@ extern "C" int cns_batch_create(cns_solver *const *members, int n, cns_batch **o
         }
     }
     for (BatchGroup &g : b->groups) {
+        g.pencil = default_batch_pencil(g);
         int rc = upload(b, g, g.pencil, false);
         if (rc) return bail(rc);
     }
