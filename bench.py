@@ -18,9 +18,11 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Gpt-RKsteps/s + %HBM roofline, FP64 vs FP32-store; ensemble p50/p99 solve latency"
 HBM_PEAK_GBS = 8000.0
-# algorithmic HBM words per grid point of one classic-RK4 step (4 stages:
-# 15 + 25 + 25 + 20 words; state resident, read and write once per stage)
-RK4_WORDS = 85
+# algorithmic HBM words per grid point of one classic-RK4 step (4 stages;
+# state resident, read and write once per stage): 15 + 25 + 25 + 20 words with
+# an accumulator in every stage (FP32 storage), 10 + 15 + 25 + 15 with one
+# formed in the third stage (FP64 storage)
+RK4_WORDS = {4: 85, 8: 65}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_k_rhs_tgv256_o8_rk4_fp64.txt")
 
 
@@ -293,11 +295,11 @@ def main():
         sol.profile_enable(False)
         sol.close()
         per_launch_ms = kms / max(launches, 1)
-        bytes_per_launch = RK4_WORDS * wsize * pts / 4.0
+        bytes_per_launch = RK4_WORDS[wsize] * wsize * pts / 4.0
         return {"ms": ms, "wall": wall, "value": pts * a.steps / (ms / 1e3) / 1e9, "pencil": pencil,
                 "per_launch_ms": per_launch_ms, "launches": launches,
                 "achieved": bytes_per_launch / (per_launch_ms / 1e3) / 1e9,
-                "step_gbs": RK4_WORDS * wsize * pts * a.steps / (ms / 1e3) / 1e9}
+                "step_gbs": RK4_WORDS[wsize] * wsize * pts * a.steps / (ms / 1e3) / 1e9}
 
     def fp32_error(nsteps):
         """Relative L2 / Linf per conserved variable of the FP32-storage state

@@ -1279,6 +1279,9 @@ static int stage_setup(const cns_solver *s, int cur, int st, bool last_visc, Par
     } else {
         // classic RK4 with an accumulator set: acc = q0 + dt/6 k1 + dt/3 k2 + dt/3 k3,
         // q = acc + dt/6 k4.  Sets: A = current, B/D stage inputs, C accumulator.
+        // FP64 storage forms acc in the third stage from the stage states B and
+        // D (stage_update); FP32 storage, whose stage states carry no low part,
+        // adds to it in each of the first three.
         const int sa = cur, sb = (cur + 1) % 4, scc = (cur + 2) % 4, sd = (cur + 3) % 4;
         const int ins[4] = {sa, sb, sd, sb}, outs[4] = {sb, sd, sb, sa};
         in = ins[st];
@@ -1292,7 +1295,15 @@ static int stage_setup(const cns_solver *s, int cur, int st, bool last_visc, Par
         // stage inputs only feed the RHS; the step result carries a low part
         A.qoutlo = as<R>(s->lo[outs[st]]);
         P.write_qlo = st == 3;
-        if (st < 3) {
+        if (!s->fp32) {
+            if (st == 2) {
+                P.write_acc = 1;
+                P.v_r = 1.0 / 3.0;
+                A.ra = as<R>(s->sets[sb]);
+                A.rb = as<R>(s->sets[sd]);
+                A.accout = as<R>(s->sets[scc]);
+            }
+        } else if (st < 3) {
             // acc = q0 + dt/6 k1, then acc += dt/3 k2, acc += dt/3 k3
             P.write_acc = 1;
             P.v_r = st == 0 ? 1.0 / 6.0 : 1.0 / 3.0;
@@ -2156,8 +2167,8 @@ static int queue_stage(cns_batch *b, const BatchGroup &g, int st) {
     const int grid = g.grid > 0 ? std::max(1, std::min(g.grid, g.nwork)) : std::max(1, g.nwork);
     BCHK(b, launch_dil_batch<R>(g.SV, g.wallx, g.nonuni, g.unitv, grid, b->stream, jobs, nm, g.nwork, g.remap));
     BLAUNCHED(b, "k_dil_batch");
-    // three update operands only in the last Kutta stage
-    const bool k3 = g.scheme == CNS_RK3_KUTTA && st == 2;
+    // three update operands only in the last Kutta stage and FP64 RK4's third
+    const bool k3 = st == 2 && (g.scheme == CNS_RK3_KUTTA || (g.scheme == CNS_RK4 && sizeof(R) == 8));
     BCHK(b, launch_rhs_batch<R>(g.S, g.SV, g.wallx, g.nonuni, g.unitv, k3, grid, b->stream, jobs, nm, g.nwork,
                                 g.remap));
     BLAUNCHED(b, "k_rhs_batch");

@@ -27,7 +27,8 @@ struct Params {
     int tile_x;  // x width of the launch's tiles (16 or 32; host dispatch of the dilatation kernel)
     // stage update, per conserved field:
     //   q_out   = s1 + dt (w_ra ra + w_rb rb + w_r rhs)   (when write_q)
-    //   acc_out = s2 + dt (v_r rhs)                       (when write_acc)
+    //   acc_out = s2 + dt (v_r rhs)                       (when write_acc; FP64
+    //             storage: rb + v_r (ra - rb + dt rhs), RK4's third stage)
     //   r_out   = rhs                                     (when write_r)
     int write_q, use_ra, use_rb, write_acc, write_r;
     int comp;       // FP32 storage: the state carries a compensation (low) part
@@ -65,7 +66,7 @@ struct StagePtrs {
     const R *dil;  // dilatation of qin (one field)
     const R *s1;   // state term of the update (stage input, step-start state or accumulator)
     const R *ra;   // previous rhs (low-storage RK3 r_prev; Kutta k1)
-    const R *rb;   // Kutta k2
+    const R *rb;   // Kutta k2 (RK4's third stage, FP64: ra, rb the first two stage states)
     const R *s2;   // state term of the accumulator update (RK4)
     R *qout;       // updated state
     R *rout;       // right-hand side output

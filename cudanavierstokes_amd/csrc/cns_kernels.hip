@@ -32,8 +32,9 @@ static hipError_t go_rhs_v(bool wallx, bool nonuni, int nb, hipStream_t st, cons
 
 template <typename R, int S, int SV>
 static hipError_t go_rhs(bool wallx, bool nonuni, int nb, hipStream_t st, const Params &P, const StagePtrs<R> &A) {
-    // three update operands only in the last Kutta stage (q0, k1, k2)
-    const bool k3 = P.use_ra && P.use_rb;
+    // three update operands only in the last Kutta stage (q0, k1, k2) and, with
+    // FP64 storage, RK4's third (q0, q1, q2)
+    const bool k3 = (P.use_ra && P.use_rb) || (sizeof(R) == 8 && P.write_acc);
     if (P.unit_visc)
         return k3 ? go_rhs_v<R, S, SV, true, true>(wallx, nonuni, nb, st, P, A)
                   : go_rhs_v<R, S, SV, true, false>(wallx, nonuni, nb, st, P, A);

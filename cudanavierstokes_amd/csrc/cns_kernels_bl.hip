@@ -24,7 +24,7 @@ static hipError_t go_rhs_bl_v(bool nonuni, int nb, hipStream_t st, const Params 
 
 template <int S, int SV>
 static hipError_t go_rhs_bl(bool nonuni, int nb, hipStream_t st, const Params &P, const StagePtrs<double> &A) {
-    const bool k3 = P.use_ra && P.use_rb;
+    const bool k3 = (P.use_ra && P.use_rb) || P.write_acc;
     if (P.unit_visc)
         return k3 ? go_rhs_bl_v<S, SV, true, true>(nonuni, nb, st, P, A)
                   : go_rhs_bl_v<S, SV, true, false>(nonuni, nb, st, P, A);

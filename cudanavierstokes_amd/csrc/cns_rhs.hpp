@@ -421,18 +421,15 @@ __device__ __forceinline__ void with_flags(int key, F &f, FlagList<F0, FR...>) {
     else
         with_flags(key, f, FlagList<FR...>{});
 }
-// Stage kinds per storage type: RK4 stages 1-3 and 4; low-storage RK3
-// stages 1, 2 and 3 (Kutta's first two stages have the flags of the first
-// two); with K3 the last Kutta stage.  FP32 storage adds the compensated
-// sums (F_COMP) and the low part of the step result (F_QLO); a sponge
-// (always on in the boundary layer) adds F_SPONGE.
-template <typename R, bool K3, bool SPONGE>
+// Stage kinds of FP64 storage: RK4 stages 1, 2 and 4; low-storage RK3 stages
+// 1, 2 and 3 (Kutta's first two stages have the flags of the first two); with
+// K3 the last Kutta stage and RK4's third.  A sponge (always on in the
+// boundary layer) adds F_SPONGE.
+template <bool K3, bool SPONGE>
 struct CommonFlags {
-    static constexpr int C = Off<R>::on ? F_COMP : 0, L = Off<R>::on ? F_QLO : 0, SP = SPONGE ? F_SPONGE : 0;
-    using type = std::conditional_t<
-        K3, FlagList<F_Q | F_RA | F_RB | C | L | SP>,
-        FlagList<F_Q | F_ACC | C | SP, F_Q | C | L | SP, F_Q | F_R | C | L | SP, F_Q | F_RA | F_R | C | L | SP,
-                 F_Q | F_RA | C | L | SP>>;
+    static constexpr int SP = SPONGE ? F_SPONGE : 0;
+    using type = std::conditional_t<K3, FlagList<F_Q | F_RA | F_RB | SP, F_Q | F_ACC | SP>,
+                                    FlagList<F_Q | SP, F_Q | F_R | SP, F_Q | F_RA | F_R | SP, F_Q | F_RA | SP>>;
 };
 
 __device__ __forceinline__ long long uniform64(long long v) {
@@ -442,8 +439,9 @@ __device__ __forceinline__ long long uniform64(long long v) {
 }
 
 // Operands of one plane's stage update: s1 and a second operand, ra
-// (low-storage RK3, Kutta) or s2 (RK4's accumulator), rb as a third in the
-// last Kutta stage (K3), and on FP32 storage the low parts of the
+// (low-storage RK3, Kutta) or s2 (RK4's accumulator on FP32 storage), rb as a
+// third in the last Kutta stage and FP64 RK4's third (K3: ra and rb the two
+// stage states before), and on FP32 storage the low parts of the
 // compensated sets.  An array a stage does not use aliases the stage input,
 // so its loads are cache hits; all are loaded unconditionally.
 template <typename R>
@@ -483,7 +481,8 @@ __device__ __forceinline__ void load_ops(Arr arr, int fl, long poff, long fs, un
 // The end of one point's stage (plane k, column i, byte offset coff in the
 // plane): sponge (src/sponge.cu:31-41), the viscous CFL maximum from the
 // point's mu, then q_out = s1 + dt (w_ra ra + w_rb rb + w_r rhs),
-// acc_out = s2 + dt v_r rhs and r_out = rhs as the flags select.  With FP32
+// acc_out = s2 + dt v_r rhs (FP64: rb + v_r (ra - rb + dt rhs)) and r_out = rhs
+// as the flags select.  With FP32
 // storage the update is evaluated in FP64 on the compensated pair hi + lo and
 // rounded back to hi and lo (F_COMP).
 template <typename R, bool K3, class Arr>
@@ -566,10 +565,17 @@ __device__ __forceinline__ void stage_update(const Params &P, const StagePtrs<R>
 #pragma unroll
             for (int q = 0; q < 5; q++) st_at(ro + q * fs, coff, rhs[q]);
         }
-        if (fl & F_ACC) {
+        if (K3 && (fl & F_ACC)) {
+            // RK4, third stage: the step's sum q0 + dt/6 k1 + dt/3 (k2 + k3)
+            // from the two stage states q1 = q0 + dt/2 k1, q2 = q0 + dt/2 k2,
+            //   q2 + ((q1 - q2) + dt k3) / 3,
+            // so that stages 1 and 2 write no accumulator and stages 2 and 3
+            // read none back: 65 words a point and step instead of 80 (25 of
+            // them written instead of 35), one rounding of the sum fewer
             R *const ao = arr(6, poff);
 #pragma unroll
-            for (int q = 0; q < 5; q++) st_at(ao + q * fs, coff, o.e2[q] + dt * (R(s_w[3]) * rhs[q]));
+            for (int q = 0; q < 5; q++)
+                st_at(ao + q * fs, coff, o.e3[q] + R(s_w[3]) * ((o.e2[q] - o.e3[q]) + dt * rhs[q]));
         }
     }
 }
@@ -1179,7 +1185,7 @@ __device__ __forceinline__ void rhs_tile_split(const Params &P, const StagePtrs<
             __syncthreads();  // z part of the last plane
             if (act && z1 > z0) finish(z1 - 1, (z1 - 1 - z0) & 1);
         };
-        with_flags(fl & ~F_VISC, march, typename CommonFlags<R, K3, BL>::type{});
+        with_flags(fl & ~F_VISC, march, typename CommonFlags<K3, BL>::type{});
     }
     if (P.want_visc_max) block_max_atomic(vmax, P.visc_max_out, red);
 }
