@@ -1337,7 +1337,10 @@ static int queue_steps_t(cns_solver *s, int nsteps, bool want_par, bool want_tim
                 hipLaunchKernelGGL(k_reset_visc, dim3(1), dim3(1), 0, s->stream, s->d_sc);
                 LAUNCHED(s, "k_reset_visc");
             }
-            hipLaunchKernelGGL(k_cfl<R>, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, s->stream, s->base, cur, vfs,
+            // four points a lane at least: below 2^20 points the launch waits
+            // for its workgroups' two atomics each (64^3: 1024 workgroups 15 us)
+            const long wgs = std::min<long>(RED_BLOCKS, (s->n + 4 * RED_THREADS - 1) / (4 * RED_THREADS));
+            hipLaunchKernelGGL(k_cfl<R>, dim3((unsigned)wgs), dim3(RED_THREADS), 0, s->stream, s->base, cur, vfs,
                                s->d_sc);
             LAUNCHED(s, "k_cfl<R>");
             hipLaunchKernelGGL(k_dt_finalize, dim3(1), dim3(1), 0, s->stream, c.cfl, s->d_sc);
@@ -1355,9 +1358,15 @@ static int queue_steps_t(cns_solver *s, int nsteps, bool want_par, bool want_tim
                                c.len_x * c.len_y * c.len_z, (double *)nullptr, (double *)nullptr, istep);
             LAUNCHED(s, "k_final");
         }
-        hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(1), 0, s->stream, s->d_sc, want_time ? s->d_time : nullptr,
-                           istep);
-        LAUNCHED(s, "k_advance_time");
+        // the steps up to the next check share this dt and, but for the boundary
+        // layer's blowing, nothing in them reads the time: one launch advances
+        // it for all of them (one a step cost 64^3 order 4 2 us of its 64)
+        if (cfl_step || c.boundary_layer) {
+            const int ahead = c.boundary_layer ? 1 : std::min(c.check_cfl, nsteps - istep);
+            hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(1), 0, s->stream, s->d_sc,
+                               want_time ? s->d_time : nullptr, istep, ahead);
+            LAUNCHED(s, "k_advance_time");
+        }
         if (what & 2) {
             hipLaunchKernelGGL(k_final, dim3(1), dim3(RED_THREADS), 0, s->stream, s->d_part, s->d_sc, 2, c.forcing_z,
                                c.len_x * c.len_y * c.len_z, s->d_par1, s->d_par2, istep);

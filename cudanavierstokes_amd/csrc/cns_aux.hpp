@@ -148,11 +148,17 @@ static __global__ void k_reset_visc(Scalars *sc) {
     if (threadIdx.x == 0 && blockIdx.x == 0) sc->visc_max = 0ull;
 }
 
-// time[istep] = time + dt (src/calc_stress.cu:12-14, src/cuda_math.cu:17-19)
-static __global__ void k_advance_time(Scalars *sc, double *time_out, int istep) {
+// time[istep + i] = time + dt (src/calc_stress.cu:12-14, src/cuda_math.cu:17-19)
+// for the n steps from istep on, which share one dt
+static __global__ void k_advance_time(Scalars *sc, double *time_out, int istep, int n) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        sc->time = sc->time + sc->dt;
-        if (time_out) time_out[istep] = sc->time;
+        const double dt = sc->dt;
+        double t = sc->time;
+        for (int i = 0; i < n; i++) {
+            t = t + dt;
+            if (time_out) time_out[istep + i] = t;
+        }
+        sc->time = t;
     }
 }
 
