@@ -1165,6 +1165,20 @@ __device__ __forceinline__ void rhs_tile_split(const Params &P, const StagePtrs<
                 if constexpr (BL) __syncthreads();  // x-top ghosts of plane k
                 if (act) {
                     if constexpr (fin) finish(k - 1, b ^ 1);
+                    // Plane k's update operands, needed after the next barrier:
+                    // issued here they have the whole plane to arrive (at its
+                    // end only the barrier's wait, with the stores before them:
+                    // order 8 / 6 at 256^3 747 -> 711 / 681 -> 638 us, order 6
+                    // at 160^3 197 -> 177, order-6 channel 199 -> 195), at the
+                    // price of their registers during the stencils, which the
+                    // order-8 general-viscosity form (227 -> 234) and the
+                    // boundary layer (1566 -> 1579) do not have.  The schedule
+                    // barrier holds only the loads in place.
+                    constexpr bool early_ops = !BL && (UNITV || S < 4);
+                    if constexpr (early_ops) {
+                        load_ops<R, K3>(arr, flx, (long)k * mxy, fs, coff, ops);
+                        __builtin_amdgcn_sched_barrier(0x3CF);
+                    }
                     const auto FX = FXb(b);
                     const auto FY = FYb(b);
                     R d1x[3], d2x[3];
@@ -1177,7 +1191,7 @@ __device__ __forceinline__ void rhs_tile_split(const Params &P, const StagePtrs<
                     dir_terms<R, S, SV, 1, false, UNITV>(P, FY, vs, xpi, g, d2y, fy);
                     wc = FX(QW, 0);
                     muc = (double)FX(QM, 0);
-                    load_ops<R, K3>(arr, flx, (long)k * mxy, fs, coff, ops);
+                    if constexpr (!early_ops) load_ops<R, K3>(arr, flx, (long)k * mxy, fs, coff, ops);
                 }
             };
             if (z0 < z1) body(z0, std::false_type{});
