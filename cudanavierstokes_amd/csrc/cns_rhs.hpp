@@ -422,14 +422,16 @@ __device__ __forceinline__ void with_flags(int key, F &f, FlagList<F0, FR...>) {
         with_flags(key, f, FlagList<FR...>{});
 }
 // Stage kinds of FP64 storage: RK4 stages 1, 2 and 4; low-storage RK3 stages
-// 1, 2 and 3 (Kutta's first two stages have the flags of the first two); with
-// K3 the last Kutta stage and RK4's third.  A sponge (always on in the
-// boundary layer) adds F_SPONGE.
+// 1, 2 and 3 (Kutta's first two stages have the flags of the first two); a
+// right-hand side alone (cns_rhs, cns_rhs_noalloc), which then loads none of
+// the ten operands the run-time form loads for every stage; with K3 the last
+// Kutta stage and RK4's third.  A sponge (always on in the boundary layer)
+// adds F_SPONGE.
 template <bool K3, bool SPONGE>
 struct CommonFlags {
     static constexpr int SP = SPONGE ? F_SPONGE : 0;
     using type = std::conditional_t<K3, FlagList<F_Q | F_RA | F_RB | SP, F_Q | F_ACC | SP>,
-                                    FlagList<F_Q | SP, F_Q | F_R | SP, F_Q | F_RA | F_R | SP, F_Q | F_RA | SP>>;
+                                    FlagList<F_Q | SP, F_Q | F_R | SP, F_Q | F_RA | F_R | SP, F_Q | F_RA | SP, F_R | SP>>;
 };
 
 __device__ __forceinline__ long long uniform64(long long v) {
