@@ -410,11 +410,12 @@ static void set_pencil(cns_solver *s, int zc) {
 // 24^3..256^3 boxes and channels, orders 4-8, both precisions, pencils
 // 1..256: 1.4-3 us a plane, fill 1-2.3 planes).  The default chunk count is
 // the one with the fewest plane times, the smaller count of equals.  Against
-// one workgroup per CU whatever the XCDs' shares (chunks of 8..256 planes):
-// the 160x128x192 order-6 channel, 4 chunks -> 3, 346 -> 202 us per launch;
-// 64^3 order 4, 8 -> 16 chunks, 22.5 -> 17.0 us; 24^3 order 6, 3 -> 24
-// chunks, 23.9 -> 12.1 us; FP32 channel, 13 -> 6 chunks, 229 -> 165 us;
-// 272x240x256, 2 -> 1 chunks, 1297 -> about 770 us.  cns_tune measures.
+// one workgroup per CU whatever the XCDs' shares (chunks of 8..256 planes),
+// with the kernel unchanged: the 160x128x192 order-6 channel, 4 chunks -> 3,
+// 346 -> 202 us per launch (195 as the kernel is now); 64^3 order 4, 8 -> 16
+// chunks, 22.5 -> 17.0 us (now 14.6); 24^3 order 6, 3 -> 24 chunks, 23.9 ->
+// 12.1 us (now 8.0); FP32 channel, 13 -> 6 chunks, 229 -> 165 us; 272x240x256,
+// 2 -> 1 chunks, 1297 -> about 770 us.  cns_tune measures.
 static int default_pencil(long cols, int nz) {
     const long xcds = 8, cus = 32, fill = 2;
     int best = nz;

@@ -326,7 +326,7 @@ __device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x
 // Viscosity law mu = T^n / Re for FP32 storage: 2^(n log2 T) with the
 // hardware base-2 logarithm and exponential (about 1 ulp each, so mu is
 // accurate to a few parts in 10^7, inside the 1e-5 budget of FP32 storage);
-// the FP64 path keeps pow.
+// the FP64 path keeps visc_pow.
 __device__ __forceinline__ float visc_law(float t, float n, float inv_re) {
     return __builtin_amdgcn_exp2f(n * __builtin_amdgcn_logf(t)) * inv_re;
 }

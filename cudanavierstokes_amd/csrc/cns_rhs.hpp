@@ -592,7 +592,9 @@ __device__ __forceinline__ void stage_update(const Params &P, const StagePtrs<R>
 //     the z stencils;
 //   - global loads are issued one plane ahead (window feed, halo) or at the
 //     top of the plane (stage-update operands), so their latency overlaps the
-//     stencil arithmetic.
+//     stencil arithmetic.  (Next loads before the staging, as the column role
+//     of the split form does: 666 -> 658 us at 256^3 order 8, but 69.1 -> 73.3
+//     at 128^3 order 6; not so here.)
 // With FP32 storage (R = float) the state is stored as offsets from the
 // reference state and the update is evaluated in FP64 on the compensated
 // pair hi + lo, rounded back to hi and lo (F_COMP).
@@ -811,15 +813,16 @@ __device__ __forceinline__ void rhs_tile(const Params &P, const StagePtrs<R> &A,
 //   column: push plane k+S into the window, stage plane k's interior and
 //           one halo point per lane, du/dz and dv/dz of plane k -> LDS;
 //   -- barrier --
-//   plane:  update of plane k-1 (its z part came through LDS), x part and
-//           y part of plane k;
+//   plane:  loads of plane k's update operands, update of plane k-1 (its z
+//           part came through LDS), x part and y part of plane k;
 //   column: z part of plane k -> LDS, window shift.
-// The plane role is the critical path: the column role takes all the work
-// that crosses no role boundary (the staging; measured: the plane role
-// waited at the barrier 3% of its time and the column role 52% with the
-// halo in the plane role, and moving it gained 4% at order 8 and 12% on
-// the order-6 channel; moving y stresses or the update instead, which
-// then cross through LDS, measured slower).  Each role takes the velocity
+// The plane role is the critical path (at 256^3 order 8 it waits at the
+// barrier 9% of its time, the column role 29%): the column role takes all the
+// work that crosses no role boundary (the staging, which gained 4% at order 8
+// and 12% on the order-6 channel; moving y stresses or the update, which
+// then cross through LDS, measured slower, and so did three roles for x, y
+// and z: 1370 against 805 us).  During a 256^3 launch the card clocks down to
+// 1.9 GHz (2.3 at 128^3).  Each role takes the velocity
 // derivatives it needs from LDS itself.  Exchange buffers and the staged
 // planes are double buffered by plane parity.  Both roles run the same
 // barriers; the role is uniform within a wave.  The sums follow rhs_tile:
